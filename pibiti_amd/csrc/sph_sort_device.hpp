@@ -40,6 +40,17 @@ __device__ __forceinline__ uint32_t block_incl_scan(uint32_t v, uint32_t* s_wave
     return v + add;
 }
 
+// Before a block lets other blocks know that its part is done: every wave
+// waits for its own stores and atomics, then the block meets.  A barrier alone
+// does not wait for them, and the fence that follows in one thread covers that
+// thread's wave only; once they are all in the L2, that one fence writes the L2
+// back for the whole block (sixteen fences, one a wave, are sixteen
+// write-backs).
+__device__ __forceinline__ void finish_block() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+}
+
 // Look-back words: (epoch << 32) | value, written once per sort and pass.
 __device__ __forceinline__ uint64_t ld_status(const uint64_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -163,8 +174,7 @@ __device__ __forceinline__ bool hist_tile(SortShared& S, uint32_t tile, uint32_t
     const uint32_t mine = hist[t / kRadix][t % kRadix];
     if (mine) atomicAdd(&counts[t], mine);
     // the last tile scans: every count is in before its tile is counted done
-    // (one fence for the block after the barrier: a fence writes back the L2)
-    __syncthreads();
+    finish_block();
     if (t == 0) {
         __threadfence();
         S.word = atomicAdd(&ctl[kCtlHistDone], 1u);
@@ -371,7 +381,7 @@ __device__ __forceinline__ void sort_slots(SortShared& S, const SlotSort& a, con
                 a.keys0[id] = nkey[e];
                 a.vals0[id] = (uint32_t)e;
             }
-            __syncthreads();
+            finish_block();
             if (t == 0) {
                 __threadfence();
                 atomicAdd(&ctl[kCtlFilled], 1u);
@@ -379,7 +389,7 @@ __device__ __forceinline__ void sort_slots(SortShared& S, const SlotSort& a, con
         } else if (w < 2 * tiles) {
             wait_for(&ctl[kCtlFilled], tiles, a.err);
             if (hist_tile<1>(S, w - tiles, tiles, a.keys0, n, a.bits, a.counts, a.offsets, ctl)) {
-                __syncthreads();
+                finish_block();
                 if (t == 0) {
                     __threadfence();
                     atomicExch(&ctl[kCtlReady], 1u);
@@ -395,7 +405,7 @@ __device__ __forceinline__ void sort_slots(SortShared& S, const SlotSort& a, con
             pass_tile<false>(S, tile, tiles, first_epoch + p, odd ? a.keys1 : a.keys0, odd ? a.vals1 : a.vals0,
                              odd ? a.keys0 : a.keys1, odd ? a.vals0 : a.vals1, n, 8 * p, digit_bits(a.bits, p),
                              a.offsets + p * kRadix, a.status, a.err);
-            __syncthreads();
+            finish_block();
             if (t == 0) {
                 __threadfence();
                 atomicAdd(&ctl[kCtlPass + p], 1u);
