@@ -431,13 +431,15 @@ struct ListEntries {
 
 // A lane's pair entries on their way to its group-major list: a ring in LDS
 // that leaves as 16-byte stores of four.  kByRow: looked at once per row of
-// cells, whose entries (at most 12 at kMaskCap candidates a cell) fit beside
-// three left over; else after every group of candidates.  The lanes of a
+// cells, whose entries (at kMaskCap candidates a cell at most 12, and in FAST
+// mode 13 of the particle's own row) fit beside three left over; else after
+// every group of candidates.  The lanes of a
 // wave fill up at different times, so a look after every group goes through
 // the store nearly every time for some lane.
 template <bool kByRow, int kLanes>
 struct PairRing {
     static constexpr uint32_t kSlots = kByRow ? 16u : 4u;
+    static_assert(!kByRow || 3u + own_row_entries(kMaskCap) <= kSlots, "a row beside three left over");
     uint32_t* slot0;
     uint32_t count = 0, flushed = 0, pairs = 0;
     __device__ __forceinline__ explicit PairRing(uint32_t* ring) : slot0(ring + threadIdx.x) {}

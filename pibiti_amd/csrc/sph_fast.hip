@@ -21,7 +21,8 @@
 // write per group rather than per pair.  Entries are
 // group-major (entries 4g .. 4g + 3 of slot i in the uint4 at g n + i) and
 // there is room for every group the capped walk can produce (27 cells of at
-// most ceil(max_par_in_cell / 4) groups), so the lists never overflow.  The
+// most ceil(max_par_in_cell / 4) groups, and one more where the particle
+// splits its own row's run: list_entries), so the lists never overflow.  The
 // count word of a slot holds the entries (low 16 bits) and the pairs (high
 // 16 bits).
 #include "sph_device.hpp"
@@ -196,7 +197,7 @@ inline uint32_t blocks_for(uint32_t n) { return n == 0 ? 1u : (n + kBlock - 1) /
 uint32_t fast_list_groups(uint32_t max_par_in_cell, uint32_t n) {
     const uint32_t least = n <= kRowGatherMax ? kMaskCap : 0u;  // a row lane's list has room for full cells
     const uint32_t cap = max_par_in_cell < least ? least : max_par_in_cell;
-    return (27u * ((cap + 3u) / 4u) + 3u) / 4u;
+    return list_groups(cap);
 }
 
 hipError_t launch_density_fast(const LaunchCfg& c, const StepBuffers& b, float4* rec, uint4* nbr, uint32_t* nnb,

@@ -253,6 +253,31 @@ hipError_t launch_extra_terms(const LaunchCfg& c, const StepBuffers& b, float4* 
 // groups, counts in nnb) and force record (rec: 2 float4 per slot);
 // launch_force then walks those entries with the fast arithmetic.
 constexpr uint32_t kFastMaxCap = 64;
+// Most entries a particle's own row can leave in FAST mode: three full cells,
+// each a run of candidates of its own or one run with its neighbours, and the
+// run with the particle split there, which can take one group of four more
+// than the cells do (47 others of 3 x 16 as 17 + 30 are 5 + 8 groups).
+constexpr uint32_t own_row_entries(uint32_t cap) {
+    uint32_t most = 0;
+    for (uint32_t merged = 0; merged < 4; ++merged)  // bit 0: with the cell before it, bit 1: with the one after
+        for (uint32_t at = 0; at < cap; ++at) {
+            const uint32_t before = at + (merged & 1u ? cap : 0u);
+            const uint32_t after = cap - 1u - at + (merged & 2u ? cap : 0u);
+            const uint32_t alone = (merged & 1u ? 0u : 1u) + (merged & 2u ? 0u : 1u);
+            const uint32_t e = (before + 3u) / 4u + (after + 3u) / 4u + alone * ((cap + 3u) / 4u);
+            most = e > most ? e : most;
+        }
+    return most;
+}
+// Entries the lists of a walk of 27 cells have room for, and their uint4s.
+constexpr uint32_t list_entries(uint32_t cap) { return 27u * ((cap + 3u) / 4u) + 1u; }
+constexpr uint32_t list_groups(uint32_t cap) { return (list_entries(cap) + 3u) / 4u; }
+constexpr bool lists_hold_the_walk() {
+    for (uint32_t cap = 1; cap <= kFastMaxCap; ++cap)
+        if (24u * ((cap + 3u) / 4u) + own_row_entries(cap) > list_entries(cap)) return false;
+    return true;
+}
+static_assert(lists_hold_the_walk(), "the pair lists have room for every group of the capped walk");
 uint32_t fast_list_groups(uint32_t max_par_in_cell, uint32_t n);
 // Whether the step's gathers go through the pair entries (then each slot's
 // count word holds its force pairs): FAST always, the other orders while

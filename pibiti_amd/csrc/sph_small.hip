@@ -37,7 +37,7 @@ using namespace dev;
 
 constexpr int kRows = 9;
 constexpr uint32_t kRowEntries = 3u * ((kMaskCap + 3u) / 4u);  // 12: three cells of at most kMaskCap slots
-static_assert(kRows * kRowEntries <= 4u * ((27u * ((kMaskCap + 3u) / 4u) + 3u) / 4u), "rows fit the entry lists");
+static_assert(kRows * kRowEntries <= 4u * list_groups(kMaskCap), "rows fit the entry lists");
 static_assert(kRowEntries % 4u == 0u, "whole uint4 groups per row");
 static_assert(kRows <= 4 * kMaskWords, "the lanes' pair counts fit the mask words");
 
