@@ -626,6 +626,15 @@ int sph_debug_fail_alloc(uint32_t after);
  * patterns; C row-major float.  Synchronous, uses device 0.               */
 int sph_mfma_selftest(int variant, const uint16_t* a, const uint16_t* b, float* c);
 
+/* Self-test of the force's pair scale, the short exact root, reciprocal and
+ * quotient beside the general IEEE sequences (no counterpart in the
+ * reference).  par: h, Spiky factor, minDist, minDens; r2, psum = p_i + p_j
+ * and rr = rho_i rho_j of n pairs.  fast and general receive, for pair k, the
+ * pressure term at 2k and the kernel-density product at 2k + 1; in_range[k]
+ * is 1 where the step would keep the fast pair.  Synchronous, device 0.    */
+int sph_pair_selftest(uint32_t n, const float par[4], const float* r2, const float* psum, const float* rr,
+                      float* fast, float* general, uint32_t* in_range);
+
 /* ------------------------------------------------------------------------ */
 /* Learned pair-force surrogate (extension; no counterpart in the reference).
  * For every neighbour pair of particle i (|x_i - x_j| < h, j != i, the

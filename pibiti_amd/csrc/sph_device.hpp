@@ -96,26 +96,29 @@ __device__ __forceinline__ float sqrt_ieee(float x) {
 //   quotient    q = a y with y the rounded 1 / b, moved by (a - b q) y
 //               (Markstein, "Computation of elementary functions on the IBM
 //               RISC System/6000 processor", 1990).
-// On this hardware the root was compared with the IEEE one for every mantissa
-// of both exponent parities, the reciprocal for every mantissa, and the
-// quotient for every pair of mantissas whose quotient lies within 7 units of
-// the product's last place of a rounding boundary (40,702,450 pairs; farther
-// ones cannot round the wrong way) and 1.7e10 random ones: no difference.
-// That takes 18 operations fewer than the compiler's general sequences, which
+// On this hardware the root agrees with the IEEE one for every mantissa of
+// both exponent parities, the reciprocal for every mantissa, and the quotient
+// wherever it lies close to a rounding boundary (within 7 units of the
+// product's last place for 2.7 million divisors; farther ones cannot round the
+// wrong way) and at random (test_pair_scale_gpu.py).
+// That takes 19 operations fewer than the compiler's general sequences, which
 // rescale their operands.  Here nothing is rescaled, so the operands have to
 // stay clear of underflow and overflow: PairRange keeps the smallest and
 // largest magnitude that matter over the pairs of an iteration (as unsigned
-// integers: a NaN counts as too large), and an iteration out of range takes
-// the general sequences (pair_scale_ieee).
+// integers: a NaN or a negative product counts as too large), and an iteration
+// out of range takes the general sequences (pair_scale_ieee).
 struct PairScale {
     float h, spiky, min_dist, min_dens;
 };
 
+// In range: r2, |a| = |((h - r) Spiky) (p_i + p_j)| and rho_i rho_j, all in
+// [2^-60, 2^96).  Then 2^-30 <= r < 2^48, so that the quotient and its residual
+// stay between 2^-108 and 2^126.  r may also be minDist, whose square is held
+// to the same 2^96: the scene's part, where the largest starts.
 struct PairRange {
-    uint32_t lo = 0x7F800000u, hi = 0u;
-    // r2 >= 2^-90 and |a| in [2^-90, 2^96), rho_i rho_j < 2^96 (a smaller one
-    // only has to give at least minDens, which it does)
-    __device__ __forceinline__ bool ok() const { return lo >= (127u - 90u) << 23 && hi < (127u + 96u) << 23; }
+    uint32_t lo = 0x7F800000u, hi;
+    __device__ __forceinline__ explicit PairRange(const PairScale& c) : hi(__float_as_uint(c.min_dist * c.min_dist)) {}
+    __device__ __forceinline__ bool ok() const { return lo >= (127u - 60u) << 23 && hi < (127u + 96u) << 23; }
 };
 
 __device__ __forceinline__ void pair_scale(const PairScale& c, float r2, float psum, float rr, PairRange& g,
@@ -123,7 +126,7 @@ __device__ __forceinline__ void pair_scale(const PairScale& c, float r2, float p
     const float y = __builtin_amdgcn_rsqf(r2);
     const float s0 = r2 * y;
     const float s = __builtin_fmaf(__builtin_fmaf(-s0, s0, r2), 0.5f * y, s0);
-    const float r = s >= c.min_dist ? s : c.min_dist;
+    const float r = fmaxf(c.min_dist, s);
     const float cc = c.h - r;
     const float a = (cc * c.spiky) * psum;
     const float z0 = __builtin_amdgcn_rcpf(r);
@@ -132,10 +135,10 @@ __device__ __forceinline__ void pair_scale(const PairScale& c, float r2, float p
     pterm = __builtin_fmaf(__builtin_fmaf(-r, q, a), z, q);
     const float w0 = __builtin_amdgcn_rcpf(rr);
     const float w = __builtin_fmaf(__builtin_fmaf(-rr, w0, 1.0f), w0, w0);
-    cd = cc * (w <= c.min_dens ? w : c.min_dens);
+    cd = cc * fminf(c.min_dens, w);
     const uint32_t ua = __float_as_uint(a) & 0x7FFFFFFFu;
-    g.lo = min(min(g.lo, ua), __float_as_uint(r2));
-    g.hi = max(max(g.hi, ua), __float_as_uint(rr));
+    g.lo = min(min(min(g.lo, ua), __float_as_uint(rr)), __float_as_uint(r2));
+    g.hi = max(max(max(g.hi, ua), __float_as_uint(rr)), __float_as_uint(r2));
 }
 
 __device__ __forceinline__ void pair_scale_ieee(const PairScale& c, float r2, float psum, float rr, float& pterm,

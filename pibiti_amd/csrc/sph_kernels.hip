@@ -1774,7 +1774,7 @@ __global__ __launch_bounds__(kForceBlock) void k_force_entries(
             vq[k] = rec[2 * (size_t)j[k] + 1];
         }
         float gx[kForcePairs], gy[kForcePairs], gz[kForcePairs];
-        PairRange range;
+        PairRange range(c);
         auto term = [&](const float4& xj, const float4& vj, float& tx, float& ty, float& tz, auto ieee) {
             const float rx = xi.x - xj.x, ry = xi.y - xj.y, rz = xi.z - xj.z;
             const float r2 = rx * rx + ry * ry + rz * rz;

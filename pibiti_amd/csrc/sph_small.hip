@@ -279,7 +279,7 @@ __global__ __launch_bounds__(64) void k_force_rows(sph_params one, const sph_par
                 xq[u] = rec[2 * (size_t)j[u]];
                 vq[u] = rec[2 * (size_t)j[u] + 1];
             }
-            PairRange range;
+            PairRange range(c);
             auto term = [&](int u, const float4& xj, const float4& vj, auto ieee) {
                 const float rx = xi.x - xj.x, ry = xi.y - xj.y, rz = xi.z - xj.z;
                 const float r2 = rx * rx + ry * ry + rz * rz;
@@ -412,4 +412,52 @@ hipError_t launch_force_rows(const LaunchCfg& c, const StepBuffers& b, float4* v
     return hipGetLastError();
 }
 
+namespace {
+
+// The pair scale of n pairs by both sequences (sph_pair_selftest).
+__global__ __launch_bounds__(256) void k_pair_selftest(uint32_t n, PairScale c, const float* __restrict__ in,
+                                                       float2* __restrict__ fast, float2* __restrict__ general,
+                                                       uint32_t* __restrict__ in_range) {
+    const uint32_t k = blockIdx.x * 256u + threadIdx.x;
+    if (k >= n) return;
+    const float r2 = in[k], psum = in[(size_t)n + k], rr = in[2 * (size_t)n + k];
+    PairRange range(c);
+    float2 f, g;
+    pair_scale(c, r2, psum, rr, range, f.x, f.y);
+    pair_scale_ieee(c, r2, psum, rr, g.x, g.y);
+    fast[k] = f;
+    general[k] = g;
+    in_range[k] = range.ok() ? 1u : 0u;
+}
+
+}  // namespace
 }  // namespace sph
+
+extern "C" int sph_pair_selftest(uint32_t n, const float par[4], const float* r2, const float* psum, const float* rr,
+                                 float* fast, float* general, uint32_t* in_range) {
+    if (!par || !r2 || !psum || !rr || !fast || !general || !in_range || n > (1u << 26))
+        return SPH_ERR_INVALID_ARGUMENT;
+    int ndev = 0;
+    if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) return SPH_ERR_NO_DEVICE;
+    if (n == 0) return SPH_OK;
+    const size_t row = (size_t)n * sizeof(float);
+    void* mem = nullptr;  // r2, psum, rr, in_range | fast | general
+    hipError_t e = sph::device_malloc(&mem, 8 * row);
+    if (e != hipSuccess) return e == hipErrorOutOfMemory ? SPH_ERR_OUT_OF_MEMORY : SPH_ERR_DEVICE;
+    char* m = static_cast<char*>(mem);
+    const float* in[3] = {r2, psum, rr};
+    for (int k = 0; k < 3 && e == hipSuccess; ++k) e = hipMemcpy(m + k * row, in[k], row, hipMemcpyHostToDevice);
+    const size_t at = 4 * row;  // (a multiple of 16: the pairs are aligned)
+    if (e == hipSuccess) {
+        const sph::dev::PairScale c{par[0], par[1], par[2], par[3]};
+        hipLaunchKernelGGL(sph::k_pair_selftest, dim3((n + 255u) / 256u), dim3(256), 0, 0, n, c,
+                           reinterpret_cast<const float*>(m), reinterpret_cast<float2*>(m + at),
+                           reinterpret_cast<float2*>(m + at + 2 * row), reinterpret_cast<uint32_t*>(m + 3 * row));
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpy(in_range, m + 3 * row, row, hipMemcpyDeviceToHost);
+    if (e == hipSuccess) e = hipMemcpy(fast, m + at, 2 * row, hipMemcpyDeviceToHost);
+    if (e == hipSuccess) e = hipMemcpy(general, m + at + 2 * row, 2 * row, hipMemcpyDeviceToHost);
+    (void)hipFree(mem);
+    return e == hipSuccess ? SPH_OK : SPH_ERR_DEVICE;
+}

@@ -363,6 +363,7 @@ SIGNATURES = {
     "sph_batch_autotune": (C.c_int, [_P, C.c_char_p, _up, _fp]),
     "sph_batch_info": (C.c_int, [_P, _up, _up, _up, _up]),
     "sph_mfma_selftest": (C.c_int, [C.c_int, C.POINTER(C.c_uint16), C.POINTER(C.c_uint16), _fp]),
+    "sph_pair_selftest": (C.c_int, [C.c_uint32, _fp, _fp, _fp, _fp, _fp, _fp, _up]),
     "sph_model_create": (C.c_int, [C.c_int, C.POINTER(MlpNorm), C.c_uint64, C.POINTER(_P)]),
     "sph_model_destroy": (C.c_int, [_P]),
     "sph_model_get_norm": (C.c_int, [_P, C.POINTER(MlpNorm)]),
