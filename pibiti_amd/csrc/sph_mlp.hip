@@ -516,7 +516,7 @@ __global__ __launch_bounds__(kBlk, 2) void k_mlp_bwd(const MlpArgs a) {
     // fragments read again in every tile
     __shared__ bf16x8 s_w2n[8 * 64];   // -W2, lane = output unit
     __shared__ bf16x8 s_w2tf[8 * 64];  // W2 columns
-    __shared__ bf16x8 s_b2n[2 * 64];   // -b2 in two BF16 parts (k slots 0 and 1 of lane half 0)
+    __shared__ bf16x8 s_b2n[2 * 64];   // -b2 in three BF16 parts, all of its 24 bits (k slots 0 to 2 of lane half 0)
     __shared__ bf16x8 s_ident[2 * 64];
     __shared__ float4 s_w3[kOut][kHid / 4];
     __shared__ float s_db[kWaves * kGroup * kRowStride];
@@ -534,8 +534,11 @@ __global__ __launch_bounds__(kBlk, 2) void k_mlp_bwd(const MlpArgs a) {
         u32x4 w = {0u, 0u, 0u, 0u};
         if (g == 0) {
             const float b = -a.params[kOffB2 + 32 * t + p];
-            const __bf16 hi = bf(b);
-            w[0] = cvt2((float)hi, b - (float)hi);
+            const float hi = (float)bf(b);
+            const float rest = fabsf(hi) < __builtin_huge_valf() ? b - hi : 0.0f;
+            const float mid = (float)bf(rest);
+            w[0] = cvt2(hi, mid);
+            w[1] = cvt2(rest - mid, 0.0f);
         }
         s_b2n[threadIdx.x] = __builtin_bit_cast(bf16x8, w);
         s_ident[threadIdx.x] = unit_identity(t, g, p);
@@ -595,7 +598,8 @@ __global__ __launch_bounds__(kBlk, 2) void k_mlp_bwd(const MlpArgs a) {
             rn = ps.load(jn);
             jn = ps.index(t + 2);
             const bf16x8 E = edge_features(g, valid, rc, kc, nm);
-            const u32x4 ow = {valid && g == 0 ? 0x3f803f80u : 0u, 0u, 0u, 0u};
+            const uint32_t ones = valid && g == 0 ? 0x3f803f80u : 0u;
+            const u32x4 ow = {ones, ones, 0u, 0u};
             const bf16x8 bias_b = __builtin_bit_cast(bf16x8, ow);
 
             bf16x8 h1t[4];
