@@ -615,7 +615,9 @@ int sph_debug_poke(sph_ctx* ctx, int what, uint32_t index, uint32_t value);
 
 /* Testing hook (no counterpart in the reference): makes the library's
  * after-th device allocation from now on fail with SPH_ERR_OUT_OF_MEMORY,
- * as a full device would (after = 1: the next one); 0 disarms it.  It fires
+ * as a full device would (after = 1: the next one); 0 disarms it.  A read
+ * of an array counts as one more, the pinned buffer it goes through: where
+ * that one fails, the read takes the runtime's copies instead.  It fires
  * once and disarms itself.  Process-wide.                                  */
 int sph_debug_fail_alloc(uint32_t after);
 

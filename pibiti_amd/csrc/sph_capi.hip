@@ -14,11 +14,18 @@ namespace {
 std::atomic<uint32_t> fail_alloc_countdown{0};
 }  // namespace
 
-hipError_t device_malloc(void** ptr, size_t bytes) {
+namespace {
+// The sph_debug_fail_alloc count passes one allocation: whether it is to fail.
+bool allocation_fails() {
     uint32_t k = fail_alloc_countdown.load();
     while (k > 0 && !fail_alloc_countdown.compare_exchange_weak(k, k - 1)) {
     }
-    if (k == 1) {
+    return k == 1;
+}
+}  // namespace
+
+hipError_t device_malloc(void** ptr, size_t bytes) {
+    if (allocation_fails()) {
         *ptr = nullptr;
         return hipErrorOutOfMemory;
     }
@@ -26,32 +33,21 @@ hipError_t device_malloc(void** ptr, size_t bytes) {
 }
 
 namespace {
-std::mutex stage_mu;  // guards the three below; stage_taken: a transfer uses the buffer
+std::mutex stage_mu;  // guards the two below; stage_taken: a transfer uses the buffer
 char* stage_mem = nullptr;
 bool stage_taken = false;
-uint32_t stage_users = 0;
 }  // namespace
 
-void host_stage_add_user() {
-    std::lock_guard<std::mutex> lock(stage_mu);
-    ++stage_users;
-}
-
-void host_stage_remove_user() {
-    std::lock_guard<std::mutex> lock(stage_mu);
-    // (a transfer belongs to a live engine, so the last one leaves none)
-    if (--stage_users == 0 && stage_mem) {
-        (void)hipHostFree(stage_mem);
-        stage_mem = nullptr;
-    }
-}
-
+// The memory is coherent: a kernel's writes go to it and stay in no cache of
+// the GPU.  (A buffer that is only portable is not: the runtime gives
+// coarse-grained memory for that flag alone, which the GPU's L2s hold until
+// their next system-wide write-back.)
 HostStage::HostStage() {
     std::lock_guard<std::mutex> lock(stage_mu);
-    if (stage_taken) return;
+    if (stage_taken || allocation_fails()) return;
     if (!stage_mem) {
         void* p = nullptr;
-        if (hipHostMalloc(&p, kHostStageBytes + 64, hipHostMallocPortable) != hipSuccess) {
+        if (hipHostMalloc(&p, kHostStageBytes + 64, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
             (void)hipGetLastError();
             return;
         }

@@ -94,12 +94,12 @@ inline uint32_t bits_for(uint64_t cells) {
 using namespace detail;
 
 // One pinned host buffer for the process's small transfers (sph_capi.hip):
-// allocated at the first one, freed with the last engine.  A transfer holds it
+// 1 MiB, allocated at the first one and held until the process ends, as the
+// allocation-free sort's scratch is.  A transfer holds it
 // from its first copy to the end of its use; a second thread finds it taken
-// and copies through the runtime's own staging instead.
+// and copies through the runtime's own staging instead, as every transfer does
+// where the buffer cannot be allocated.
 constexpr size_t kHostStageBytes = 1u << 20;
-void host_stage_add_user();
-void host_stage_remove_user();
 class HostStage {
 public:
     HostStage();  // takes the buffer if it is free
@@ -229,11 +229,6 @@ struct Engine {
         graph = nullptr;
         graph_steps = 0;
     }
-
-    Engine() { host_stage_add_user(); }
-    ~Engine() { host_stage_remove_user(); }
-    Engine(const Engine&) = delete;
-    Engine& operator=(const Engine&) = delete;
 
     void release() {
         drop_graph();

@@ -1,5 +1,6 @@
 """Shared pytest setup: repo root on sys.path, the `gpu` marker, helpers."""
 import os
+import subprocess
 import sys
 from pathlib import Path
 
@@ -9,10 +10,32 @@ import pytest
 ROOT = Path(__file__).resolve().parent.parent
 if str(ROOT) not in sys.path:
     sys.path.insert(0, str(ROOT))
+if str(ROOT / "tests") not in sys.path:
+    sys.path.insert(0, str(ROOT / "tests"))
+
+
+_launcher = None
 
 
 def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs a HIP device (MI355X); run with -m gpu")
+    global _launcher
+    if os.path.exists("/dev/kfd"):
+        from child_launcher import Launcher
+        _launcher = Launcher()
+
+
+def pytest_unconfigure(config):
+    if _launcher:
+        _launcher.close()
+
+
+@pytest.fixture(autouse=True)
+def children_from_the_helper(request, monkeypatch):
+    """GPU tests launch their children from a process that never uses the GPU
+    (child_launcher.py says why)."""
+    if _launcher and request.node.get_closest_marker("gpu"):
+        monkeypatch.setattr(subprocess, "run", _launcher.run)
 
 
 @pytest.fixture(scope="session")
