@@ -62,7 +62,7 @@ __global__ __launch_bounds__(kSortBlock) void k_pass(const uint32_t* __restrict_
         if (S.word == gridDim.x - 1) ctl[kCtlPass + pass] = 0u;
     }
     __syncthreads();
-    pass_tile<true>(S, S.word, gridDim.x, epoch, in, nullptr, out, nullptr, n, 8 * pass, digit_bits(bits, pass),
+    pass_tile<true>(S, S.word, epoch, in, nullptr, out, nullptr, n, 8 * pass, digit_bits(bits, pass),
                     offsets + pass * kRadix, status, err);
 }
 
@@ -76,12 +76,12 @@ uint32_t radix_num_tiles(uint32_t n) {
 namespace {
 
 // Scratch layout: digit counts | digit offsets | control words | look-back
-// words (a count and a span sum per tile and digit).
+// words (one per tile and digit).
 constexpr size_t kDigits = (size_t)kMaxPasses * kRadix;
 constexpr size_t kHeadBytes = 2 * kDigits * 4 + kCtlNum * 4;
 static_assert(kHeadBytes % 8 == 0, "the status words are 8 bytes each");
 
-constexpr size_t scratch_bytes_for_tiles(uint64_t tiles) { return kHeadBytes + 2 * (size_t)tiles * kRadix * 8; }
+constexpr size_t scratch_bytes_for_tiles(uint64_t tiles) { return kHeadBytes + (size_t)tiles * kRadix * 8; }
 
 void carve(RadixSortPlan& plan, uint32_t n, void* scratch) {
     plan.n = n;
@@ -148,7 +148,7 @@ constexpr size_t kNoAllocBytes = sph::scratch_bytes_for_tiles((kNoAllocMaxPairs 
 constexpr int kMaxDevices = 64;
 
 // The allocation-free sort's scratch: one copy per GPU, held until the
-// process ends (about 0.8 MB).  Host code uses the per-device address from
+// process ends (about 0.5 MB).  Host code uses the per-device address from
 // hipGetSymbolAddress (noalloc_ptr), never this name.
 __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 static_assert(kNoAllocBytes % 4 == 0, "cleared by words");

@@ -51,7 +51,15 @@ __device__ __forceinline__ void finish_block() {
     __syncthreads();
 }
 
-// Look-back words: (epoch << 32) | value, written once per sort and pass.
+// Look-back words, one per tile and digit: (epoch << 32) | kSpanKnown |
+// (span sum << kSpanShift) | tile count.  A tile writes its word twice in a
+// pass, first with its count and then with its span sum (at most kSpan kTile)
+// beside it: one word for both halves what the sort's scratch holds.
+constexpr uint32_t kCountMask = (1u << 13) - 1u;
+constexpr uint32_t kSpanShift = 13, kSpanMask = (1u << 17) - 1u;
+constexpr uint32_t kSpanKnown = 1u << 30;
+static_assert(kTile <= kCountMask && kSpan * kTile <= kSpanMask, "counts and span sums fit their fields");
+
 __device__ __forceinline__ uint64_t ld_status(const uint64_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -59,9 +67,10 @@ __device__ __forceinline__ void st_status(uint64_t* p, uint32_t epoch, uint32_t 
     __hip_atomic_store(p, ((uint64_t)epoch << 32) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Sum of digit d's words of the tiles tile - k stride (k = 1 .. count, all
-// >= 0) that thread q of the digit's kLook takes (k = q + 1, q + 1 + kLook,
-// ...), waiting for each to carry the epoch.
+// Sum of digit d's counts (kSpans: span sums) of the tiles tile - k stride
+// (k = 1 .. count, all >= 0) that thread q of the digit's kLook takes (k =
+// q + 1, q + 1 + kLook, ...), waiting for each to be written.
+template <bool kSpans>
 __device__ __forceinline__ uint32_t look_back(const uint64_t* __restrict__ words, uint32_t tile, uint32_t stride,
                                               uint32_t count, int d, int q, uint32_t epoch,
                                               uint32_t* __restrict__ err) {
@@ -73,11 +82,12 @@ __device__ __forceinline__ uint32_t look_back(const uint64_t* __restrict__ words
 #pragma unroll
             for (int u = 0; u < kBatch; ++u) {
                 const uint32_t k = k0 + (uint32_t)(u * kLook);
-                w[u] = (uint64_t)epoch << 32;
+                w[u] = (uint64_t)epoch << 32 | kSpanKnown;
                 if (k <= count) w[u] = ld_status(words + (size_t)(tile - k * stride) * kRadix + d);
             }
 #pragma unroll
-            for (int u = 0; u < kBatch; ++u) waiting = waiting || (uint32_t)(w[u] >> 32) != epoch;
+            for (int u = 0; u < kBatch; ++u)
+                waiting = waiting || (uint32_t)(w[u] >> 32) != epoch || (kSpans && ((uint32_t)w[u] & kSpanKnown) == 0u);
             if (!waiting) break;
             if (++spins > kSpinLimit) {
                 atomicOr(err, 1u);
@@ -86,7 +96,8 @@ __device__ __forceinline__ uint32_t look_back(const uint64_t* __restrict__ words
             __builtin_amdgcn_s_sleep(1);
         }
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u) sum += (uint32_t)w[u];
+        for (int u = 0; u < kBatch; ++u)
+            sum += kSpans ? ((uint32_t)w[u] >> kSpanShift) & kSpanMask : (uint32_t)w[u] & kCountMask;
     }
     return sum;
 }
@@ -194,7 +205,7 @@ __device__ __forceinline__ bool hist_tile(SortShared& S, uint32_t tile, uint32_t
 // pairs (keys_in / keys_out; the others unused) instead of a key array and a
 // value array.
 template <bool kPairs>
-__device__ __forceinline__ void pass_tile(SortShared& S, uint32_t tile, uint32_t tiles, uint32_t epoch,
+__device__ __forceinline__ void pass_tile(SortShared& S, uint32_t tile, uint32_t epoch,
                                           const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in,
                                           uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out,
                                           uint32_t n, uint32_t shift, uint32_t pass_bits,
@@ -267,20 +278,19 @@ __device__ __forceinline__ void pass_tile(SortShared& S, uint32_t tile, uint32_t
     // Look back: the counts of the kSpan - 1 tiles before this one make its
     // span sum, which is published; the span sums of every kSpan-th tile
     // before it add up to the rest.  kLook threads per digit.
-    uint64_t* const spans = status + (size_t)tiles * kRadix;
     const int d = t % kRadix, q = t / kRadix;
     const uint32_t near = tile < kSpan - 1u ? tile : kSpan - 1u;  // tiles before it in its span
-    S.look[q][d] = look_back(status, tile, 1u, near, d, q, epoch, err);
+    S.look[q][d] = look_back<false>(status, tile, 1u, near, d, q, epoch, err);
     __syncthreads();
     uint32_t prefix = 0;
     if (t < kRadix) {
 #pragma unroll
         for (int u = 0; u < kLook; ++u) prefix += S.look[u][t];
-        st_status(spans + (size_t)tile * kRadix + t, epoch, prefix + cnt);
+        st_status(status + (size_t)tile * kRadix + t, epoch, kSpanKnown | (prefix + cnt) << kSpanShift | cnt);
     }
     if (tile >= (uint32_t)kSpan) {  // (the same for the whole block)
         __syncthreads();
-        S.look[q][d] = look_back(spans, tile, kSpan, tile / kSpan, d, q, epoch, err);
+        S.look[q][d] = look_back<true>(status, tile, kSpan, tile / kSpan, d, q, epoch, err);
         __syncthreads();
         if (t < kRadix) {
 #pragma unroll
@@ -402,7 +412,7 @@ __device__ __forceinline__ void sort_slots(SortShared& S, const SlotSort& a, con
             else
                 wait_for(&ctl[kCtlPass + p - 1], tiles, a.err);
             const bool odd = (p & 1u) != 0;
-            pass_tile<false>(S, tile, tiles, first_epoch + p, odd ? a.keys1 : a.keys0, odd ? a.vals1 : a.vals0,
+            pass_tile<false>(S, tile, first_epoch + p, odd ? a.keys1 : a.keys0, odd ? a.vals1 : a.vals0,
                              odd ? a.keys0 : a.keys1, odd ? a.vals0 : a.vals1, n, 8 * p, digit_bits(a.bits, p),
                              a.offsets + p * kRadix, a.status, a.err);
             finish_block();
