@@ -1435,13 +1435,12 @@ __global__ __launch_bounds__(kBlock) void k_density_tiled(
 // a FAST-mode surrogate step: 48 us (57 with the counters added up by every
 // block), against 77 us for the ring form and 9 us
 // for the two kernels that followed it.
-template <bool kBatch>
+// (One scene: the surrogate steps no batches.)
 __global__ __launch_bounds__(kBlock) void k_density_lists(
-    sph_params one, const sph_params* __restrict__ tab, const uint32_t* __restrict__ sid, uint32_t n,
-    const float4* __restrict__ pos, const float* __restrict__ xyz, const uint32_t* __restrict__ cell_start,
-    const uint32_t* __restrict__ cell_end, float2* __restrict__ rhop, uint32_t* __restrict__ nbr,
-    uint32_t* __restrict__ nnb, uint32_t* __restrict__ counters, float inv_rho0, uint32_t* ticket,
-    unsigned long long* part, double* __restrict__ dev_out, uint32_t first, uint32_t ncopy,
+    sph_params one, uint32_t n, const float4* __restrict__ pos, const float* __restrict__ xyz,
+    const uint32_t* __restrict__ cell_start, const uint32_t* __restrict__ cell_end, float2* __restrict__ rhop,
+    uint32_t* __restrict__ nbr, uint32_t* __restrict__ nnb, uint32_t* __restrict__ counters, float inv_rho0,
+    uint32_t* ticket, unsigned long long* part, double* __restrict__ dev_out, uint32_t first, uint32_t ncopy,
     uint32_t* __restrict__ cnt_out) {
     const uint32_t b0 = xcd_tile(blockIdx.x, gridDim.x), i = b0 * kBlock + threadIdx.x;
     uint32_t listed = 0, over = 0;
@@ -1449,8 +1448,8 @@ __global__ __launch_bounds__(kBlock) void k_density_lists(
     if (i < n) {
         const PosPacked src{xyz};
         const uint32_t c =
-            density_one<kBatch, SPH_PREC_REFERENCE, true, PosPacked, false, false, false, false, true>(
-                i, one, tab, sid, pos, cell_start, cell_end, rhop, n, nbr, nnb, counters, &src);
+            density_one<false, SPH_PREC_REFERENCE, true, PosPacked, false, false, false, false, true>(
+                i, one, nullptr, nullptr, pos, cell_start, cell_end, rhop, n, nbr, nnb, counters, &src);
         listed = min(c, kNbrCap);
         over = c > kNbrCap ? 1u : 0u;
         dev = fabs((double)rhop[i].x * (double)inv_rho0 - 1.0);
@@ -2363,22 +2362,16 @@ hipError_t launch_density_lists(const LaunchCfg& c, const StepBuffers& b, uint32
 // The entries' LDS slots hold a row of cells at kMaskCap candidates a cell;
 // compensated sums add hits under a branch, where the entries save nothing.
 bool density_report_lists(const LaunchCfg& c, const StepBuffers& b) {
-    return c.tune[3] == 0 && b.xyz && c.max_cap <= kMaskCap && c.precision != SPH_PREC_KAHAN;
+    return !c.tab && c.tune[3] == 0 && b.xyz && c.max_cap <= kMaskCap && c.precision != SPH_PREC_KAHAN;
 }
 
 hipError_t launch_density_lists(const LaunchCfg& c, const StepBuffers& b, uint32_t* nbr, uint32_t* nnb,
                                 const DensityReport& r, hipStream_t s) {
     if (!density_report_lists(c, b)) return hipErrorInvalidValue;
     const dim3 grid(blocks_for(c.n, kBlock)), block(kBlock);
-    auto* part = reinterpret_cast<unsigned long long*>(r.part);
-    if (c.tab)
-        hipLaunchKernelGGL((k_density_lists<true>), grid, block, 0, s, c.one, c.tab, b.sid_cur, c.n, b.pos_cur, b.xyz,
-                           b.cell_start, b.cell_end, b.rhop, nbr, nnb, b.counters, r.inv_rho0, r.ticket, part, r.dev,
-                           r.first, r.ncopy, r.counts);
-    else
-        hipLaunchKernelGGL((k_density_lists<false>), grid, block, 0, s, c.one, c.tab, b.sid_cur, c.n, b.pos_cur,
-                           b.xyz, b.cell_start, b.cell_end, b.rhop, nbr, nnb, b.counters, r.inv_rho0, r.ticket, part,
-                           r.dev, r.first, r.ncopy, r.counts);
+    hipLaunchKernelGGL(k_density_lists, grid, block, 0, s, c.one, c.n, b.pos_cur, b.xyz, b.cell_start, b.cell_end,
+                       b.rhop, nbr, nnb, b.counters, r.inv_rho0, r.ticket,
+                       reinterpret_cast<unsigned long long*>(r.part), r.dev, r.first, r.ncopy, r.counts);
     return hipGetLastError();
 }
 
