@@ -99,7 +99,7 @@ __device__ __forceinline__ float sqrt_ieee(float x) {
 // On this hardware the root agrees with the IEEE one for every mantissa of
 // both exponent parities, the reciprocal for every mantissa, and the quotient
 // wherever it lies close to a rounding boundary (within 7 units of the
-// product's last place for 2.7 million divisors; farther ones cannot round the
+// product's last place for 2.7 million quotients; farther ones cannot round the
 // wrong way) and at random (test_pair_scale_gpu.py).
 // That takes 19 operations fewer than the compiler's general sequences, which
 // rescale their operands.  Here nothing is rescaled, so the operands have to
@@ -112,9 +112,11 @@ struct PairScale {
 };
 
 // In range: r2, |a| = |((h - r) Spiky) (p_i + p_j)| and rho_i rho_j, all in
-// [2^-60, 2^96).  Then 2^-30 <= r < 2^48, so that the quotient and its residual
-// stay between 2^-108 and 2^126.  r may also be minDist, whose square is held
-// to the same 2^96: the scene's part, where the largest starts.
+// [2^-60, 2^96), and a zero a (a scene without pressure: 0 of either sign over
+// r is that 0 here too; 1,048,576 particles 391 -> 307 us a step).  Then 2^-30
+// <= r < 2^48, so that the quotient and its residual stay between 2^-108 and
+// 2^126.  r may also be minDist, whose square is held to the same 2^96: the
+// scene's part, where the largest starts.
 struct PairRange {
     uint32_t lo = 0x7F800000u, hi;
     __device__ __forceinline__ explicit PairRange(const PairScale& c) : hi(__float_as_uint(c.min_dist * c.min_dist)) {}
@@ -132,12 +134,12 @@ __device__ __forceinline__ void pair_scale(const PairScale& c, float r2, float p
     const float z0 = __builtin_amdgcn_rcpf(r);
     const float z = __builtin_fmaf(__builtin_fmaf(-r, z0, 1.0f), z0, z0);
     const float q = a * z;
-    pterm = __builtin_fmaf(__builtin_fmaf(-r, q, a), z, q);
+    pterm = __builtin_fmaf(-__builtin_fmaf(r, q, -a), z, q);
     const float w0 = __builtin_amdgcn_rcpf(rr);
     const float w = __builtin_fmaf(__builtin_fmaf(-rr, w0, 1.0f), w0, w0);
     cd = cc * fminf(c.min_dens, w);
     const uint32_t ua = __float_as_uint(a) & 0x7FFFFFFFu;
-    g.lo = min(min(min(g.lo, ua), __float_as_uint(rr)), __float_as_uint(r2));
+    g.lo = min(min(min(g.lo, ua - 1u), __float_as_uint(rr)), __float_as_uint(r2));  // (zero: the largest)
     g.hi = max(max(max(g.hi, ua), __float_as_uint(rr)), __float_as_uint(r2));
 }
 

@@ -136,3 +136,14 @@ def test_ordinary_pairs_stay_in_range():
     r2 = (h * rng.random(n) ** (1 / 3)).astype(np.float32) ** 2
     par = (h, -45.0 / (np.pi * h ** 6), 0.005, 1e-6)
     check(par, r2, rng.normal(0, 3000, n).astype(np.float32), rng.uniform(1e5, 4e6, n).astype(np.float32), least=0.999)
+
+
+def test_pairs_without_pressure_stay_in_range():
+    """Stiffness 0: the pressure sum is a zero of either sign."""
+    rng = np.random.default_rng(13)
+    n, h = 100_000, 0.02
+    r2 = (h * rng.random(n) ** (1 / 3)).astype(np.float32) ** 2
+    zero = np.where(rng.random(n) < 0.5, np.float32(0.0), np.float32(-0.0)).astype(np.float32)
+    for spiky in (-45.0 / (np.pi * h ** 6), 45.0 / (np.pi * h ** 6)):
+        g = check((h, spiky, 0.005, 1e-6), r2, zero, rng.uniform(1e5, 4e6, n).astype(np.float32), least=0.999)
+        assert not np.any(g[:, 0])
