@@ -58,8 +58,8 @@ __global__ __launch_bounds__(kSortBlock) void k_pass(const uint32_t* __restrict_
                                                      uint32_t* __restrict__ err) {
     __shared__ SortShared S;
     if (threadIdx.x == 0) {
-        S.word = atomicAdd(&ctl[kCtlPass + pass], 1u);
-        if (S.word == gridDim.x - 1) ctl[kCtlPass + pass] = 0u;
+        S.word = atomicAdd(&ctl[kCtlPass + pass * kLine], 1u);
+        if (S.word == gridDim.x - 1) ctl[kCtlPass + pass * kLine] = 0u;
     }
     __syncthreads();
     pass_tile<true>(S, S.word, epoch, in, nullptr, out, nullptr, n, 8 * pass, digit_bits(bits, pass),

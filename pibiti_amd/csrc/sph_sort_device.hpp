@@ -19,7 +19,8 @@ constexpr int kMaxPasses = 4;
 constexpr int kLook = kSortBlock / kRadix;  // threads per digit in the look-back
 constexpr int kSpan = 16;                   // tiles a span sum covers
 constexpr int kBatch = 4;                   // look-back loads in flight per thread
-constexpr uint32_t kSpinLimit = 1u << 22;
+constexpr uint32_t kSpinLimit = 1u << 22;    // of a look-back, some tenths of a second
+constexpr uint32_t kWaitLimit = 1u << 19;    // of wait_for, about half a second
 
 
 // Inclusive scan of one value per thread over the block: a shuffle scan in
@@ -40,16 +41,18 @@ __device__ __forceinline__ uint32_t block_incl_scan(uint32_t v, uint32_t* s_wave
     return v + add;
 }
 
-// Before a block lets other blocks know that its part is done: every wave
-// waits for its own stores and atomics, then the block meets.  A barrier alone
-// does not wait for them, and the fence that follows in one thread covers that
-// thread's wave only; once they are all in the L2, that one fence writes the L2
-// back for the whole block (sixteen fences, one a wave, are sixteen
-// write-backs).
+// Hand-over between the blocks of one launch.  Before a block lets other blocks
+// know that its part is done, every wave waits for its own stores and atomics,
+// then the block meets (finish_block): a barrier alone does not wait for them,
+// and a thread's fence covers its own wave only.  Atomics are then in memory;
+// stores are in the XCC's L2, which one thread writes back (release_agent).
+// The receiving block's one thread that waits acquires before its block meets.
 __device__ __forceinline__ void finish_block() {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
 }
+__device__ __forceinline__ void release_agent() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent"); }
+__device__ __forceinline__ void acquire_agent() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
 
 // Look-back words, one per tile and digit: (epoch << 32) | kSpanKnown |
 // (span sum << kSpanShift) | tile count.  A tile writes its word twice in a
@@ -102,19 +105,26 @@ __device__ __forceinline__ uint32_t look_back(const uint64_t* __restrict__ words
     return sum;
 }
 
-// The sort's control words (RadixSortPlan::ctl), all zero between sorts but
-// the epoch.
+// The sort's control words (RadixSortPlan::ctl), all zero between sorts but the
+// epoch.  Each word that many blocks update or wait for has a cache line of
+// its own: in one line their polls and updates queue up behind each other.
+constexpr int kLine = 32;  // words
+constexpr int kStages = 1 + kMaxPasses;
+constexpr int kXccs = 16;  // values of the XCC id register
 enum Ctl : int {
-    kCtlEpoch = 0,    // sorts finished by sort_slots
-    kCtlErr = 1,      // a wait hit its bound (the plan may name another word)
-    kCtlHistDone = 2, // histogram tiles finished
-    kCtlTicket = 3,   // sort_slots: (stage, tile) tickets
-    kCtlRetired = 4,  // sort_slots: blocks that found no ticket
-    kCtlReady = 5,    // sort_slots: the digit offsets are written
-    kCtlFilled = 6,   // sort_slots: input tiles written
-    kCtlPass = 8,     // [kMaxPasses] k_pass: tile tickets; sort_slots: tiles finished
-    kCtlNum = 16
+    kCtlEpoch = 0,            // sorts finished by sort_slots
+    kCtlErr = 1,              // a wait hit its bound (the plan may name another word)
+    kCtlHistDone = 1 * kLine, // histogram tiles finished
+    kCtlTicket = 2 * kLine,   // sort_slots: (stage, tile) tickets
+    kCtlRetired = 3 * kLine,  // sort_slots: blocks that found no ticket
+    kCtlReady = 4 * kLine,    // sort_slots: the digit offsets are written
+    kCtlPass = 5 * kLine,     // [kMaxPasses] k_pass: tile tickets
+    kCtlDone = kCtlPass + kMaxPasses * kLine,     // [kStages] sort_slots: tiles whose output is in memory
+    kCtlXcc = kCtlDone + kStages * kLine,         // [kStages][kXccs] sort_slots: XccWord
+    kCtlNum = kCtlXcc + kStages * kXccs * kLine
 };
+// A stage's tiles on one XCC: taken, finished, and of these written back.
+enum XccWord : int { kXccTaken = 0, kXccFinished = 1, kXccWritten = 2 };
 
 struct SortShared {
     uint32_t wcount[kWaves][kRadix];
@@ -186,17 +196,14 @@ __device__ __forceinline__ bool hist_tile(SortShared& S, uint32_t tile, uint32_t
     if (mine) atomicAdd(&counts[t], mine);
     // the last tile scans: every count is in before its tile is counted done
     finish_block();
-    if (t == 0) {
-        __threadfence();
-        S.word = atomicAdd(&ctl[kCtlHistDone], 1u);
-    }
+    if (t == 0) S.word = atomicAdd(&ctl[kCtlHistDone], 1u);
     __syncthreads();
     if (S.word != tiles - 1) return false;
     const uint32_t c = __hip_atomic_exchange(&counts[t], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // an inclusive scan over all passes' digits; a pass's offsets are relative
     // to the passes before it, whose counts sum to n each
     const uint32_t incl = block_incl_scan<kSortBlock>(c, S.s_wave);
-    offsets[t] = incl - c - (uint32_t)(t / kRadix) * n;
+    __hip_atomic_store(&offsets[t], incl - c - (uint32_t)(t / kRadix) * n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (t == 0) ctl[kCtlHistDone] = 0u;
     return true;
 }
@@ -297,7 +304,8 @@ __device__ __forceinline__ void pass_tile(SortShared& S, uint32_t tile, uint32_t
             for (int u = 0; u < kLook; ++u) prefix += S.look[u][t];
         }
     }
-    if (t < kRadix) S.gbase[t] = digit_off[t] + prefix;
+    if (t < kRadix)
+        S.gbase[t] = __hip_atomic_load(&digit_off[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + prefix;
     __syncthreads();
 
 #pragma unroll
@@ -335,15 +343,43 @@ __device__ __forceinline__ void wait_for(const uint32_t* word, uint32_t want, ui
     if (threadIdx.x == 0) {
         uint32_t spins = 0;
         while (__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != want) {
-            if (++spins > kSpinLimit) {
+            if (++spins > kWaitLimit) {
                 atomicOr(err, 1u);
                 break;
             }
-            __builtin_amdgcn_s_sleep(2);
+            __builtin_amdgcn_s_sleep(32);
         }
+        acquire_agent();
     }
     __syncthreads();
-    __threadfence();
+}
+
+// A tile of a stage is finished (finish_block is behind it): its output is
+// counted done once it is in memory.  A write-back covers the whole L2, and
+// each one walks it: 32 tiles of an XCC that end together, each with its own,
+// take several times their own work.  So the one that leaves no taken tile
+// behind on its XCC writes back for all that finished there before it.
+// (1,048,576 particles, the place kernel of a step with the full sort: a
+// write-back and an acquire in every wave 880 us, in one wave a tile 340, with
+// the control words in lines of their own 207, one an XCC 117; a launch for
+// each stage, which every step would pay for, 148.)
+__device__ __forceinline__ void count_done(uint32_t* ctl, uint32_t stage, uint32_t xcc) {
+    uint32_t* const x = ctl + kCtlXcc + (stage * kXccs + xcc) * kLine;
+    uint32_t finished = atomicAdd(&x[kXccFinished], 1u) + 1u;
+    // counted before the taken ones are read (the last to finish has to see
+    // every one; its own was counted before its work)
+    asm volatile("" : "+v"(finished)::"memory");
+    if (finished != __hip_atomic_load(&x[kXccTaken], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+    const uint32_t written = atomicMax(&x[kXccWritten], finished);
+    if (written >= finished) return;
+    release_agent();
+    atomicAdd(&ctl[kCtlDone + stage * kLine], finished - written);
+}
+
+// The XCC (and so the L2) this wave runs on.
+__device__ __forceinline__ uint32_t xcc_id() {
+    constexpr int kHwRegXccId = 20;
+    return __builtin_amdgcn_s_getreg(kHwRegXccId | (0 << 6) | ((4 - 1) << 11)) & (kXccs - 1);
 }
 
 // The whole sort of the slots by (the low `bits` bits of nkey, original
@@ -351,10 +387,10 @@ __device__ __forceinline__ void wait_for(const uint32_t* word, uint32_t want, ui
 // this.  Its input is made here, (key, slot) in original-index order into
 // (keys0, vals0), so that a step that needs no sort does not write it; the
 // passes ping-pong with (keys1, vals1), where keys1 may be nkey.  Tickets: the
-// input tiles, the histogram tiles, then the tiles of pass 0, 1, ...; a block
-// takes the next one until none is left and waits for the last pass.  Tickets
-// are held by running blocks only, so every wait ends whatever else runs on
-// the GPU.  Returns with the sorted pairs visible to the block.
+// tiles of the input and its digit counts, then those of pass 0, 1, ...; a
+// block takes the next one until none is left and waits for the last pass.
+// Tickets are held by running blocks only, so every wait ends whatever else
+// runs on the GPU.  Returns with the sorted pairs visible to the block.
 struct SlotSort {
     uint32_t* keys0;
     uint32_t* vals0;
@@ -375,63 +411,52 @@ __device__ __forceinline__ void sort_slots(SortShared& S, const SlotSort& a, con
     // read before this block's first ticket; the last block to retire, which
     // raises it, does so after every block's last wait
     const uint32_t first_epoch = ctl[kCtlEpoch] * kMaxPasses + 1u;
+    const uint32_t xcc = xcc_id();
     for (;;) {
-        if (t == 0) S.word = atomicAdd(&ctl[kCtlTicket], 1u);
+        if (t == 0) {
+            const uint32_t w = atomicAdd(&ctl[kCtlTicket], 1u);
+            if (w < tiles * (passes + 1)) atomicAdd(&ctl[kCtlXcc + (w / tiles * kXccs + xcc) * kLine + kXccTaken], 1u);
+            S.word = w;
+        }
         __syncthreads();
         const uint32_t w = S.word;
         __syncthreads();
-        if (w >= tiles * (passes + 2)) break;
-        if (w < tiles) {
+        if (w >= tiles * (passes + 1)) break;
+        const uint32_t stage = w / tiles, tile = w % tiles;
+        if (stage == 0) {
 #pragma unroll
             for (int it = 0; it < kItems; ++it) {
-                const uint64_t e = (uint64_t)w * kTile + (uint64_t)it * kSortBlock + t;
+                const uint64_t e = (uint64_t)tile * kTile + (uint64_t)it * kSortBlock + t;
                 if (e >= n) continue;
                 const uint32_t id = pid[e];
                 if (id >= n) continue;
                 a.keys0[id] = nkey[e];
                 a.vals0[id] = (uint32_t)e;
             }
-            finish_block();
-            if (t == 0) {
-                __threadfence();
-                atomicAdd(&ctl[kCtlFilled], 1u);
-            }
-        } else if (w < 2 * tiles) {
-            wait_for(&ctl[kCtlFilled], tiles, a.err);
-            if (hist_tile<1>(S, w - tiles, tiles, a.keys0, n, a.bits, a.counts, a.offsets, ctl)) {
+            if (hist_tile<1>(S, tile, tiles, nkey, n, a.bits, a.counts, a.offsets, ctl)) {
                 finish_block();
-                if (t == 0) {
-                    __threadfence();
-                    atomicExch(&ctl[kCtlReady], 1u);
-                }
+                if (t == 0) atomicExch(&ctl[kCtlReady], 1u);
             }
         } else {
-            const uint32_t p = w / tiles - 2, tile = w % tiles;
-            if (p == 0)
-                wait_for(&ctl[kCtlReady], 1u, a.err);
-            else
-                wait_for(&ctl[kCtlPass + p - 1], tiles, a.err);
+            const uint32_t p = stage - 1;
+            wait_for(&ctl[kCtlDone + p * kLine], tiles, a.err);
+            if (p == 0) wait_for(&ctl[kCtlReady], 1u, a.err);
             const bool odd = (p & 1u) != 0;
             pass_tile<false>(S, tile, first_epoch + p, odd ? a.keys1 : a.keys0, odd ? a.vals1 : a.vals0,
                              odd ? a.keys0 : a.keys1, odd ? a.vals0 : a.vals1, n, 8 * p, digit_bits(a.bits, p),
                              a.offsets + p * kRadix, a.status, a.err);
             finish_block();
-            if (t == 0) {
-                __threadfence();
-                atomicAdd(&ctl[kCtlPass + p], 1u);
-            }
         }
+        if (t == 0) count_done(ctl, stage, xcc);
         __syncthreads();
     }
-    if (passes)
-        wait_for(&ctl[kCtlPass + passes - 1], tiles, a.err);
-    else
-        wait_for(&ctl[kCtlFilled], tiles, a.err);  // one cell: the input is the result
-    if (t == 0 && atomicAdd(&ctl[kCtlRetired], 1u) == gridDim.x - 1) {
-        // every other block is past its last use of the control words
-        for (int c = kCtlHistDone; c < kCtlNum; ++c) ctl[c] = 0u;
-        ctl[kCtlEpoch] += 1u;
-    }
+    wait_for(&ctl[kCtlDone + passes * kLine], tiles, a.err);
+    if (t == 0) S.word = atomicAdd(&ctl[kCtlRetired], 1u);
+    __syncthreads();
+    if (S.word != gridDim.x - 1) return;
+    // every other block is past its last use of the control words
+    for (int c = kLine + t; c < kCtlNum; c += kSortBlock) ctl[c] = 0u;
+    if (t == 0) ctl[kCtlEpoch] += 1u;
 }
 
 }  // namespace sortdev

@@ -45,3 +45,22 @@ def test_full_sorts_over_many_tiles(make, passes):
             if step == 0:
                 o = oracle.step_f32(p, pos, vel)
                 assert np.array_equal(s.get_array(sph.SPH_ARRAY_POSITION), o["pos"])
+
+
+def test_more_tiles_than_blocks_at_once():
+    """2,195,200 particles: 536 tiles a stage, more than the 512 blocks that
+    run at a time, on two consecutive steps."""
+    p, pos, vel = scenes.scaled_dam_break((140, 112, 140), seed=53, vel_sigma=2.0)[:3]
+    wmin, cs = np.array(p.world_min, np.float64), np.array(p.cell_size, np.float64)
+    centre = wmin + (np.floor((pos[0, :3] - wmin) / cs) + 0.5) * cs
+    rng = np.random.default_rng(7)
+    pos[:5000, :3] = (centre + rng.uniform(-0.002, 0.002, (5000, 3))).astype(np.float32)
+    vel[:5000] = 0
+    print("case: full sort, 536 tiles", flush=True)
+    with sph.SphSystem(p) as s:
+        s.reset(pos, vel)
+        for step in range(2):
+            s.update(1)
+            st = s.stats()
+            assert st["full_sort"] == 1 and st["sort_errors"] == 0, step
+            assert_sorted_like_oracle(s, p)
