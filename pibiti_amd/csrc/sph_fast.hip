@@ -203,7 +203,10 @@ uint32_t fast_list_groups(uint32_t max_par_in_cell, uint32_t n) {
 hipError_t launch_density_fast(const LaunchCfg& c, const StepBuffers& b, float4* rec, uint4* nbr, uint32_t* nnb,
                                hipStream_t s) {
     if (!b.xyz) return hipErrorInvalidValue;  // the place kernel packs the positions
-    if (row_gathers_in_use(c, b)) return launch_density_rows(c, b, s);
+    if (row_gathers_in_use(c, b)) {
+        launch_density_rows(c, b, s);
+        return hipGetLastError();
+    }
     const dim3 grid(blocks_for(c.n)), block(kBlock);
     const auto launch = [&](auto batch, auto by_row) {
         hipLaunchKernelGGL((k_density_fast<decltype(batch)::value, decltype(by_row)::value>), grid, block, 0, s, c.one,

@@ -291,8 +291,8 @@ bool pair_entries_in_use(const LaunchCfg& c, const StepBuffers& b);
 // tune setting asks for the pair entries.
 constexpr uint32_t kRowGatherMax = 65536u;
 bool row_gathers_in_use(const LaunchCfg& c, const StepBuffers& b);
-hipError_t launch_density_rows(const LaunchCfg& c, const StepBuffers& b, hipStream_t s);
-hipError_t launch_force_rows(const LaunchCfg& c, const StepBuffers& b, float4* vel_out, float4* dvel, hipStream_t s);
+void launch_density_rows(const LaunchCfg& c, const StepBuffers& b, hipStream_t s);
+void launch_force_rows(const LaunchCfg& c, const StepBuffers& b, float4* vel_out, float4* dvel, hipStream_t s);
 
 hipError_t launch_density_fast(const LaunchCfg& c, const StepBuffers& b, float4* rec, uint4* nbr, uint32_t* nnb,
                                hipStream_t s);

@@ -2165,7 +2165,7 @@ template <bool kBatch, int kPrec>
 void density_impl(const LaunchCfg& c, const StepBuffers& b, hipStream_t s) {
     const uint32_t grid = c.tune[1];
     if (use_rows(c, b))
-        (void)launch_density_rows(c, b, s);
+        launch_density_rows(c, b, s);
     else if (use_entries(c, b) && c.max_cap <= kMaskCap)  // a row's entries fit the ring
         hipLaunchKernelGGL((k_density_entries<kBatch, kPrec, true>), dim3(blocks_for(c.n, kBlock)), dim3(kBlock), 0, s,
                            c.one, c.tab, b.sid_cur, c.n, b.pos_cur, b.xyz, b.vel_cur, b.cell_start, b.cell_end,
@@ -2229,7 +2229,7 @@ template <bool kBatch, int kPrec>
 void force_impl(const LaunchCfg& c, const StepBuffers& b, float4* vel_out, float4* dvel,
                 hipStream_t s) {
     if (use_rows(c, b)) {
-        (void)launch_force_rows(c, b, vel_out, dvel, s);
+        launch_force_rows(c, b, vel_out, dvel, s);
         return;
     }
     if (use_entries(c, b)) {
@@ -2402,7 +2402,7 @@ hipError_t launch_force(const LaunchCfg& c, const StepBuffers& b, float4* vel_ou
         if (!b.pairs || !b.pair_cnt || !b.rec) return hipErrorInvalidValue;
         const dim3 grid(blocks_for(c.n, kForceBlock)), block(kForceBlock);
         if (row_gathers_in_use(c, b))
-            (void)launch_force_rows(c, b, vel_out, dvel, s);
+            launch_force_rows(c, b, vel_out, dvel, s);
         else if (c.tab)
             hipLaunchKernelGGL((k_force_entries<true, SPH_PREC_FAST>), grid, block, 0, s, c.one, c.tab, b.sid_cur, c.n,
                                b.vel_cur, b.rec, b.pairs, b.pair_cnt, vel_out, dvel, b.dt_dev);

@@ -384,7 +384,7 @@ bool row_gathers_in_use(const LaunchCfg& c, const StepBuffers& b) {
            b.pair_cnt && b.rec && b.xyz;
 }
 
-hipError_t launch_density_rows(const LaunchCfg& c, const StepBuffers& b, hipStream_t s) {
+void launch_density_rows(const LaunchCfg& c, const StepBuffers& b, hipStream_t s) {
     const auto launch = [&](auto batch) {
         constexpr bool kBatch = decltype(batch)::value;
         if (c.precision == SPH_PREC_FAST)
@@ -395,10 +395,9 @@ hipError_t launch_density_rows(const LaunchCfg& c, const StepBuffers& b, hipStre
             density_rows<kBatch, SPH_PREC_REFERENCE>(c, b, s);
     };
     c.tab ? launch(std::true_type{}) : launch(std::false_type{});
-    return hipGetLastError();
 }
 
-hipError_t launch_force_rows(const LaunchCfg& c, const StepBuffers& b, float4* vel_out, float4* dvel, hipStream_t s) {
+void launch_force_rows(const LaunchCfg& c, const StepBuffers& b, float4* vel_out, float4* dvel, hipStream_t s) {
     const auto launch = [&](auto batch) {
         constexpr bool kBatch = decltype(batch)::value;
         if (c.precision == SPH_PREC_FAST)
@@ -409,7 +408,6 @@ hipError_t launch_force_rows(const LaunchCfg& c, const StepBuffers& b, float4* v
             force_rows<kBatch, SPH_PREC_REFERENCE>(c, b, vel_out, dvel, s);
     };
     c.tab ? launch(std::true_type{}) : launch(std::false_type{});
-    return hipGetLastError();
 }
 
 namespace {
