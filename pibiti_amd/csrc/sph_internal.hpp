@@ -46,7 +46,7 @@ struct RadixSortPlan {
     uint32_t* counts = nullptr;     // digit counts of every pass (zero between sorts)
     uint32_t* digit_off = nullptr;  // exclusive digit offsets per pass
     uint32_t* ctl = nullptr;        // tickets and progress counters
-    uint64_t* status = nullptr;     // look-back words, one per (tile, digit)
+    uint64_t* status = nullptr;     // look-back words
     uint32_t* err = nullptr;        // set when a wait hit its limit
 };
 

@@ -15,14 +15,16 @@
 //   pass (x bits/8)  per tile: stable local ranking with 64-lane ballots (peer
 //                 mask per digit, rank = popcount of lower peers), tile digit
 //                 counts published and prefixed across tiles by a look-back
-//                 in two levels, local reorder in LDS, coalesced runs written
-//                 to each digit's global range.
+//                 over spans of 16, of 16 spans and so on, local reorder in
+//                 LDS, coalesced runs written to each digit's global range.
 // A tile is 4096 pairs on 1024 threads, four to a thread: with 256 tiles at 1M
 // a CU has one tile, and sixteen waves rank it in a quarter of the time of
 // four.  The tiles of such a sort all publish at about the same time, so a
-// tile has to add up every count before it; span sums over 16 tiles make that
-// two short rounds of loads (a pass at 1,000,003 random keys with 256 tiles:
-// one count at a time 28 us, 64 counts a round 20.6 us, spans 14.2 us).
+// tile has to add up every count before it; sums over spans of 16 tiles, over
+// 16 spans and so on make that one short round of loads a level (a pass at
+// 1,000,003 random keys with 256 tiles: one count at a time 28 us, 64 counts a
+// round 20.6 us, spans 14.2 us; 134,217,728 pairs, three passes and the
+// histogram: 5.5 ms, with spans of tiles as the only sums 27.6 ms).
 //
 // Two forms:
 //   k_hist, k_pass  one launch each (the stand-alone sort);
@@ -62,7 +64,7 @@ __global__ __launch_bounds__(kSortBlock) void k_pass(const uint32_t* __restrict_
         if (S.word == gridDim.x - 1) ctl[kCtlPass + pass * kLine] = 0u;
     }
     __syncthreads();
-    pass_tile<true>(S, S.word, epoch, in, nullptr, out, nullptr, n, 8 * pass, digit_bits(bits, pass),
+    pass_tile<true>(S, S.word, gridDim.x, epoch, in, nullptr, out, nullptr, n, 8 * pass, digit_bits(bits, pass),
                     offsets + pass * kRadix, status, err);
 }
 
@@ -76,12 +78,14 @@ uint32_t radix_num_tiles(uint32_t n) {
 namespace {
 
 // Scratch layout: digit counts | digit offsets | control words | look-back
-// words (one per tile and digit).
+// words (a row of one per digit for each tile, for each span of tiles, ...).
 constexpr size_t kDigits = (size_t)kMaxPasses * kRadix;
 constexpr size_t kHeadBytes = 2 * kDigits * 4 + kCtlNum * 4;
 static_assert(kHeadBytes % 8 == 0, "the status words are 8 bytes each");
 
-constexpr size_t scratch_bytes_for_tiles(uint64_t tiles) { return kHeadBytes + (size_t)tiles * kRadix * 8; }
+constexpr size_t scratch_bytes_for_tiles(uint32_t tiles) {
+    return kHeadBytes + (size_t)look_back_rows(tiles) * kRadix * 8;
+}
 
 void carve(RadixSortPlan& plan, uint32_t n, void* scratch) {
     plan.n = n;

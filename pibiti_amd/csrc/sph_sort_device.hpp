@@ -17,8 +17,7 @@ constexpr int kTile = kSortBlock * kItems;  // pairs per tile
 constexpr int kRadix = 256;
 constexpr int kMaxPasses = 4;
 constexpr int kLook = kSortBlock / kRadix;  // threads per digit in the look-back
-constexpr int kSpan = 16;                   // tiles a span sum covers
-constexpr int kBatch = 4;                   // look-back loads in flight per thread
+constexpr int kSpan = 16;                   // words a sum of the look-back covers
 constexpr uint32_t kSpinLimit = 1u << 22;    // of a look-back, some tenths of a second
 constexpr uint32_t kWaitLimit = 1u << 19;    // of wait_for, about half a second
 
@@ -54,14 +53,15 @@ __device__ __forceinline__ void finish_block() {
 __device__ __forceinline__ void release_agent() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent"); }
 __device__ __forceinline__ void acquire_agent() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
 
-// Look-back words, one per tile and digit: (epoch << 32) | kSpanKnown |
-// (span sum << kSpanShift) | tile count.  A tile writes its word twice in a
-// pass, first with its count and then with its span sum (at most kSpan kTile)
-// beside it: one word for both halves what the sort's scratch holds.
-constexpr uint32_t kCountMask = (1u << 13) - 1u;
-constexpr uint32_t kSpanShift = 13, kSpanMask = (1u << 17) - 1u;
-constexpr uint32_t kSpanKnown = 1u << 30;
-static_assert(kTile <= kCountMask && kSpan * kTile <= kSpanMask, "counts and span sums fit their fields");
+// Look-back words: (epoch << 32) | value, written once per sort and pass: a
+// tile's digit counts, the sums over each kSpan tiles, over each kSpan of those
+// and so on, one level behind the other.
+constexpr uint32_t groups_of(uint32_t count) { return (count + kSpan - 1) / kSpan; }
+constexpr uint64_t look_back_rows(uint32_t tiles) {
+    uint64_t rows = tiles;
+    for (uint32_t c = tiles; c > (uint32_t)kSpan; c = groups_of(c)) rows += groups_of(c);
+    return rows;
+}
 
 __device__ __forceinline__ uint64_t ld_status(const uint64_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -70,38 +70,34 @@ __device__ __forceinline__ void st_status(uint64_t* p, uint32_t epoch, uint32_t 
     __hip_atomic_store(p, ((uint64_t)epoch << 32) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Sum of digit d's counts (kSpans: span sums) of the tiles tile - k stride
-// (k = 1 .. count, all >= 0) that thread q of the digit's kLook takes (k =
-// q + 1, q + 1 + kLook, ...), waiting for each to be written.
-template <bool kSpans>
-__device__ __forceinline__ uint32_t look_back(const uint64_t* __restrict__ words, uint32_t tile, uint32_t stride,
-                                              uint32_t count, int d, int q, uint32_t epoch,
-                                              uint32_t* __restrict__ err) {
-    uint32_t sum = 0, spins = 0;
-    for (uint32_t k0 = (uint32_t)q + 1u; k0 <= count; k0 += kBatch * kLook) {
-        uint64_t w[kBatch];
-        for (;;) {
-            bool waiting = false;
+// Sum of digit d's words of the rows row - k (k = 1 .. count, fewer than kSpan)
+// that thread q of the digit's kLook takes (k = q + 1, q + 1 + kLook, ...),
+// waiting for each to carry the epoch.
+__device__ __forceinline__ uint32_t look_back(const uint64_t* __restrict__ words, uint32_t row, uint32_t count, int d,
+                                              int q, uint32_t epoch, uint32_t* __restrict__ err) {
+    constexpr int kBatch = kSpan / kLook;  // loads in flight
+    static_assert(kSpan % kLook == 0, "one round of loads");
+    uint64_t w[kBatch];
+    for (uint32_t spins = 0;;) {
+        bool waiting = false;
 #pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
-                const uint32_t k = k0 + (uint32_t)(u * kLook);
-                w[u] = (uint64_t)epoch << 32 | kSpanKnown;
-                if (k <= count) w[u] = ld_status(words + (size_t)(tile - k * stride) * kRadix + d);
-            }
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u)
-                waiting = waiting || (uint32_t)(w[u] >> 32) != epoch || (kSpans && ((uint32_t)w[u] & kSpanKnown) == 0u);
-            if (!waiting) break;
-            if (++spins > kSpinLimit) {
-                atomicOr(err, 1u);
-                break;
-            }
-            __builtin_amdgcn_s_sleep(1);
+        for (int u = 0; u < kBatch; ++u) {
+            const uint32_t k = (uint32_t)(q + 1 + u * kLook);
+            w[u] = (uint64_t)epoch << 32;
+            if (k <= count) w[u] = ld_status(words + (size_t)(row - k) * kRadix + d);
         }
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u)
-            sum += kSpans ? ((uint32_t)w[u] >> kSpanShift) & kSpanMask : (uint32_t)w[u] & kCountMask;
+        for (int u = 0; u < kBatch; ++u) waiting = waiting || (uint32_t)(w[u] >> 32) != epoch;
+        if (!waiting) break;
+        if (++spins > kSpinLimit) {
+            atomicOr(err, 1u);
+            break;
+        }
+        __builtin_amdgcn_s_sleep(1);
     }
+    uint32_t sum = 0;
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) sum += (uint32_t)w[u];
     return sum;
 }
 
@@ -212,11 +208,11 @@ __device__ __forceinline__ bool hist_tile(SortShared& S, uint32_t tile, uint32_t
 // pairs (keys_in / keys_out; the others unused) instead of a key array and a
 // value array.
 template <bool kPairs>
-__device__ __forceinline__ void pass_tile(SortShared& S, uint32_t tile, uint32_t epoch,
+__device__ __forceinline__ void pass_tile(SortShared& S, uint32_t tile, uint32_t tiles, uint32_t epoch,
                                           const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in,
                                           uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out,
                                           uint32_t n, uint32_t shift, uint32_t pass_bits,
-                                          const uint32_t* __restrict__ digit_off, uint64_t* __restrict__ status,
+                                          const uint32_t* __restrict__ digit_off, uint64_t* status,
                                           uint32_t* __restrict__ err) {
     const int t = threadIdx.x;
     const int wave = t / kWave;
@@ -282,27 +278,33 @@ __device__ __forceinline__ void pass_tile(SortShared& S, uint32_t tile, uint32_t
     const uint32_t incl = block_incl_scan<kSortBlock>(cnt, S.s_wave);
     if (t < kRadix) S.dig_off[t] = incl - cnt;
 
-    // Look back: the counts of the kSpan - 1 tiles before this one make its
-    // span sum, which is published; the span sums of every kSpan-th tile
-    // before it add up to the rest.  kLook threads per digit.
+    // Look back, kLook threads per digit: the counts of the tiles before this
+    // one in its span, the sums of the spans before that one in its span, and
+    // so on.  The last tile of a span makes and publishes the span's sum.
     const int d = t % kRadix, q = t / kRadix;
-    const uint32_t near = tile < kSpan - 1u ? tile : kSpan - 1u;  // tiles before it in its span
-    S.look[q][d] = look_back<false>(status, tile, 1u, near, d, q, epoch, err);
-    __syncthreads();
-    uint32_t prefix = 0;
-    if (t < kRadix) {
+    uint32_t prefix = 0, total = cnt;
+    bool last = true;
+    for (uint32_t row = tile, rows = tiles;;) {
+        const uint32_t before = row % kSpan;  // (the same for the whole block)
+        if (before) {
+            S.look[q][d] = look_back(status, row, before, d, q, epoch, err);
+            __syncthreads();
+            if (t < kRadix) {
+                uint32_t sum = 0;
 #pragma unroll
-        for (int u = 0; u < kLook; ++u) prefix += S.look[u][t];
-        st_status(status + (size_t)tile * kRadix + t, epoch, kSpanKnown | (prefix + cnt) << kSpanShift | cnt);
-    }
-    if (tile >= (uint32_t)kSpan) {  // (the same for the whole block)
-        __syncthreads();
-        S.look[q][d] = look_back<true>(status, tile, kSpan, tile / kSpan, d, q, epoch, err);
-        __syncthreads();
-        if (t < kRadix) {
-#pragma unroll
-            for (int u = 0; u < kLook; ++u) prefix += S.look[u][t];
+                for (int u = 0; u < kLook; ++u) sum += S.look[u][t];
+                prefix += sum;
+                total += sum;
+            }
         }
+        status += (size_t)rows * kRadix;
+        last = last && before == kSpan - 1u;
+        if (rows <= (uint32_t)kSpan) break;
+        if (last && t < kRadix) st_status(status + (size_t)(row / kSpan) * kRadix + t, epoch, total);
+        row /= kSpan;
+        rows = groups_of(rows);
+        if (row == 0) break;
+        __syncthreads();
     }
     if (t < kRadix)
         S.gbase[t] = __hip_atomic_load(&digit_off[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + prefix;
@@ -442,7 +444,7 @@ __device__ __forceinline__ void sort_slots(SortShared& S, const SlotSort& a, con
             wait_for(&ctl[kCtlDone + p * kLine], tiles, a.err);
             if (p == 0) wait_for(&ctl[kCtlReady], 1u, a.err);
             const bool odd = (p & 1u) != 0;
-            pass_tile<false>(S, tile, first_epoch + p, odd ? a.keys1 : a.keys0, odd ? a.vals1 : a.vals0,
+            pass_tile<false>(S, tile, tiles, first_epoch + p, odd ? a.keys1 : a.keys0, odd ? a.vals1 : a.vals0,
                              odd ? a.keys0 : a.keys1, odd ? a.vals0 : a.vals1, n, 8 * p, digit_bits(a.bits, p),
                              a.offsets + p * kRadix, a.status, a.err);
             finish_block();
