@@ -591,7 +591,7 @@ int sph_radix_sort(uint32_t* pairs, uint32_t* temp, uint32_t n, uint32_t bits, v
 /* sph_radix_sort without any device allocation (no counterpart in the
  * reference): for callers that cannot allocate, such as tight serving loops
  * and harnesses that forbid hipMalloc.  Its scratch is a fixed array in
- * device memory, one per GPU, kept until the process ends (about 0.5 MB);
+ * device memory, one per GPU, kept until the process ends (about 0.6 MB);
  * n above SPH_SORT_NOALLOC_MAX is SPH_ERR_CAPACITY.  Every call on a GPU
  * uses that GPU's array, so calls on one GPU are serialised by a lock in
  * the library and each waits for its sort: they do not overlap within a

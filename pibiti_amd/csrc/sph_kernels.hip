@@ -1536,11 +1536,12 @@ __global__ __launch_bounds__(kBlock) void k_density_masks(
 
 // Density plus the force kernel's pair entries and force records
 // (density_one with kEntries), one slot per lane in XCD-ordered tiles.
-// Bound by the vector L1's return path (three 16-byte loads per four
-// candidates) and, close behind, by instruction issue: compares, selects,
-// conversions and maxima take twice an addition's 2.3 clocks, so the loop
-// keeps to additions and products, 32-bit offsets and one compare per
-// further use of a mask.  1,048,576 slots, reference order: 133 -> 127 us
+// Bound in the reference order by instruction issue with 56% of the lanes in
+// use (1,048,576 slots: 121,464 vector instructions a SIMD in the launch's
+// 400,000 clocks, 3.3 each; the vector L1 serves 0.68 accesses per CU and
+// clock, 0.82 in the FAST density).  Compares, selects, conversions and maxima
+// take twice an addition's 2.3 clocks, so the loop keeps to additions and
+// products, 32-bit offsets and one compare per further use of a mask.  1,048,576 slots, reference order: 133 -> 127 us
 // with the clamp for the maximum, the offsets for 64-bit pointers and one
 // compare of the group's bits instead of two.
 template <bool kBatch, int kPrec, bool kByRow>

@@ -152,7 +152,7 @@ constexpr size_t kNoAllocBytes = sph::scratch_bytes_for_tiles((kNoAllocMaxPairs 
 constexpr int kMaxDevices = 64;
 
 // The allocation-free sort's scratch: one copy per GPU, held until the
-// process ends (about 0.5 MB).  Host code uses the per-device address from
+// process ends (about 0.6 MB).  Host code uses the per-device address from
 // hipGetSymbolAddress (noalloc_ptr), never this name.
 __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 static_assert(kNoAllocBytes % 4 == 0, "cleared by words");
